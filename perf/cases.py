@@ -122,20 +122,27 @@ def _context():
     return _runtime
 
 
-def _quantize(generator, n, k, bits, group, spread):
-    """A random matrix quantized as MLX quantizes it: (code words, scales and biases as fp16 bits), on the host."""
+def _levels(generator, n, k, bits, group, spread):
+    """A random matrix quantized as MLX quantizes it, some rows at a time: (first row, code words, steps, lowest values)."""
     levels = (1 << bits) - 1
-    words = torch.empty((n, k * bits // 32), dtype=torch.int32)
-    scales = torch.empty((n, k // group), dtype=torch.float16)
-    biases = torch.empty((n, k // group), dtype=torch.float16)
-    shifts = torch.arange(0, 32, bits, device="cuda", dtype=torch.int32) if 32 % bits == 0 else None
     rows = max(1, (1 << 26) // k)
     for r in range(0, n, rows):
         c = min(rows, n - r)
         w = torch.randn((c, k // group, group), device="cuda", generator=generator) * spread
         low = w.amin(2, keepdim=True).half().float()
         step = ((w.amax(2, keepdim=True) - low) / levels).half().float()
-        codes = ((w - low) / step).round_().clamp_(0, levels).to(torch.int32).view(c, k)
+        yield r, ((w - low) / step).round_().clamp_(0, levels).to(torch.int32), step, low
+
+
+def _quantize(generator, n, k, bits, group, spread):
+    """The matrix as a file holds it: (code words, scales and biases as fp16 bits), on the host."""
+    words = torch.empty((n, k * bits // 32), dtype=torch.int32)
+    scales = torch.empty((n, k // group), dtype=torch.float16)
+    biases = torch.empty((n, k // group), dtype=torch.float16)
+    shifts = torch.arange(0, 32, bits, device="cuda", dtype=torch.int32) if 32 % bits == 0 else None
+    for r, codes, step, low in _levels(generator, n, k, bits, group, spread):
+        c = codes.shape[0]
+        codes = codes.view(c, k)
         if shifts is not None:
             packed = (codes.view(c, -1, 32 // bits) << shifts).sum(2, dtype=torch.int64)
         else:                                             # widths that straddle words: 32 codes fill `bits` words
@@ -150,6 +157,14 @@ def _quantize(generator, n, k, bits, group, spread):
         words[r:r + c] = packed.to(torch.int32).cpu()      # (the low 32 bits)
         scales[r:r + c], biases[r:r + c] = step.view(c, -1).half().cpu(), low.view(c, -1).half().cpu()
     return words.numpy().view(np.uint32), scales.numpy().view(np.uint16), biases.numpy().view(np.uint16)
+
+
+def _matrix(generator, case, n, k, spread=0.02):
+    """The same matrix as the numbers it stands for, in 64 bits."""
+    w = torch.empty((n, k), device="cuda", dtype=torch.float64)
+    for r, codes, step, low in _levels(generator, n, k, case["bits"], case["group"], spread):
+        w[r:r + codes.shape[0]] = (codes.double() * step.double() + low.double()).view(-1, k)
+    return w
 
 
 def _weight(state, generator, case, n, k, spread=0.02):
@@ -239,6 +254,29 @@ def run(s):
             ctx.gated_qgemm(s.gate, s.up, s.x_mlp.data_ptr(), t, s.act.data_ptr(), t, m, stream=stream)
         ctx.qgemm(s.down, s.act.data_ptr(), t, s.y.data_ptr(), t, m, stream=stream)
     return s.outputs
+
+
+def exact(case, seed):
+    """What run() returns, in 64 bits from the numbers the quantized weights stand for; the caches, whose bytes are a
+    quantization of their own, have no such value."""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    m, hidden, dtype = case["m"], case["hidden"], DTYPES[case["x"]][1]
+
+    def rows(count, width):
+        return torch.randn((count, width), device="cuda", generator=g).to(dtype).double()
+
+    if case["kind"] == "token":
+        table = _matrix(g, case, case["vocabulary"], hidden)
+        ids = torch.randint(0, case["vocabulary"], (m,), device="cuda", dtype=torch.int32, generator=g)
+        logits = table @ rows(1, hidden)[0]
+        return [table[ids.long()], logits, logits.argmax().view(1).to(torch.int32)]
+    kv, ffn = case["kv"], case["ffn"]
+    shapes = [(hidden, hidden), (kv, hidden), (kv, hidden), (hidden, hidden), (ffn, hidden), (ffn, hidden), (hidden, ffn)]
+    wq, wk, wv, wo, gate, up, down = (_matrix(g, case, n, k) for n, k in shapes)
+    x_attention, attended, x_mlp = (rows(m, hidden) for _ in range(3))
+    act = torch.nn.functional.silu(x_mlp @ gate.t()) * (x_mlp @ up.t())
+    outputs = [x_attention @ wq.t(), x_attention @ wk.t(), x_attention @ wv.t(), attended @ wo.t(), act, act @ down.t()]
+    return outputs + [None] * 4 if case["kind"] == "prompt" else outputs
 
 
 def work(case):
