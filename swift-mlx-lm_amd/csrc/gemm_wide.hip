@@ -23,8 +23,8 @@
 //     words of those four K-tiles as one more 16-byte load, and wait in registers; vmcnt is counted by hand, because
 //     the copies into LDS are invisible to the compiler's own bookkeeping;
 //   * one k-step is BM / 32 groups of two MFMAs; group q also reads activation fragment q of the NEXT k-step from LDS
-//     and dequantises a share of the next k-step's weight fragments (byte-lane convert, fp32 fma, one rounding to
-//     bf16 -- bit for bit the weights of dequant_q4_g*_bf16), so the matrix cores never wait for an operand;
+//     and dequantises a share of the next k-step's weight fragments (nibbles read as f16 subnormals by a mixed fp32 fma, one
+//     rounding to bf16 -- bit for bit the weights of dequant_q4_g*_bf16), so the matrix cores never wait for an operand;
 //   * one barrier per K-tile, in the middle of it: K-tile kt + 1 has landed for everyone, and the stage of K-tile
 //     kt - 1 is free for kt + 3;
 //   * BM = 256 where that fills the chip (one workgroup per CU, 256 accumulator registers per lane), BM = 128 elsewhere
