@@ -38,11 +38,16 @@ struct WideArgs {
     const uint32_t* seg_sz[2];
     const uint8_t* seg_blocks[2];
     void* seg_y[2];
+    uint32_t short_rows;         // 1: the last row tile is a short one (filled in at the launch)
     unsigned long long* probe;   // optional: [0] shader cycles, [1] 100 MHz ticks that workgroup 0 spent in the kernel
 };
 
 constexpr int kWideStages = 4;   // LDS stages of activations
 constexpr int kWideBN = 256;
+
+// The last 256-row tile holds at most 128 rows (and is not the only one): its workgroups multiply a quarter or half of
+// the fragments and are dispatched behind all others.
+inline bool wide_short_rows(uint32_t m, uint32_t bm) { return bm == 256 && m > bm && m % bm != 0 && m % bm <= 128; }
 
 // the kernel launch alone (tiles_m, tiles_n filled in here); activations bf16 / f16
 mi355q_status launch_wide_kernel_bf16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, bool sb_bf16, bool blocks);

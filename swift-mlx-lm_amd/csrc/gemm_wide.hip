@@ -27,6 +27,8 @@
 //     rounding to bf16 -- bit for bit the weights of dequant_q4_g*_bf16), so the matrix cores never wait for an operand;
 //   * one barrier per K-tile, in the middle of it: K-tile kt + 1 has landed for everyone, and the stage of K-tile
 //     kt - 1 is free for kt + 3;
+//   * a last 256-row tile of at most 64 or 128 rows copies and multiplies those fragments only, and its workgroups come last,
+//     on the CUs the last round of whole tiles leaves idle (gate+up 2 x 14336 at 517 fp32 rows 322 -> 297 us);
 //   * BM = 256 where that fills the chip (one workgroup per CU, 256 accumulator registers per lane), BM = 128 elsewhere
 //     (two workgroups per CU); where 256-row tiles would leave CUs idle, K goes over workgroups in parts.
 // The kernel text is gemm_wide.inl; this file chooses the shape, launches, and adds the parts of K.
@@ -124,6 +126,12 @@ void gemm_wide_force_shape(uint32_t bm, uint32_t splits) {
     g_wide_forced_splits.store(splits <= 8 ? splits : 0, std::memory_order_relaxed);
 }
 
+// Cycles per K-tile of a short tile (256-row form, at most 64 or 128 rows of it used).  Measured: 1300 to 1450 at 5 rows
+// (gate+up 4096 -> 2 x 14336 at 517 rows against 512: 160 against 108 us, fp32 297 against 204; the weights are dequantised
+// all the same).  Carried higher, because the cost of K parts below is low for wide results: with 1000 to 1600 that pair at
+// 270 fp32 rows went to two parts, 184 us against 169 in one, and q+k+v at 517 to four, 90 against 82 in two of 128 rows.
+constexpr double kWideShort64 = 1800.0, kWideShort128 = 1900.0;
+
 // Tile height and K parts.  What a wavefront spends on a K-tile depends on the tile height alone (the weights of its 64
 // columns are dequantised once per K-tile whatever the rows: about 2500 cycles at 256 rows, 1600 at 128, measured
 // under load), so 256-row tiles are the efficient ones and K is split into parts where they leave CUs idle: each part
@@ -145,13 +153,22 @@ GemmLaunchShape gemm_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_par
             const uint32_t per = (kt / 4 + splits - 1) / splits * 4;          // K-tiles a part, a multiple of four
             const uint32_t parts = (kt + per - 1) / per;
             if (parts != splits) continue;
-            const uint32_t wgs = ((m + bm - 1) / bm) * tiles_n * parts;
+            const uint32_t all = ((m + bm - 1) / bm) * tiles_n * parts;
+            const uint32_t shorts = wide_short_rows(m, bm) ? tiles_n * parts : 0, wgs = all - shorts;
             // cycles of a workgroup per K-tile, measured under load: 2500 at 256 rows (one workgroup a CU, whole rounds);
             // 1600 at 128 rows alone on its CU, 2950 for the two that share one (a last round of at most one per CU
             // runs alone)
             double cycles;
             if (bm == 256) {
                 cycles = (double)((wgs + cus - 1) / cus) * per * 2500.0;
+                // the short tiles of a cut last row: on the CUs the last round leaves idle, the
+                // others in rounds of their own
+                if (shorts) {
+                    const double each = m % bm <= 64 ? kWideShort64 : kWideShort128;
+                    const uint32_t idle = wgs % cus ? cus - wgs % cus : 0;
+                    const uint32_t beside = idle * (uint32_t)(2500.0 / each);
+                    if (shorts > beside) cycles += (double)((shorts - beside + cus - 1) / cus) * per * each;
+                }
             } else {
                 const uint32_t full = wgs / (2 * cus), rest = wgs % (2 * cus);
                 cycles = (double)full * per * 2950.0 + (rest > cus ? per * 2950.0 : rest ? per * 1600.0 : 0.0);

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
     constexpr int TM = BM / 32;                     // activation fragments = groups per k-step
     constexpr int A_STAGE = BM * 128;
     constexpr int AQ = BM / 32;                     // activation copies per wavefront and K-tile (8 rows each)
-    constexpr int CPK = AQ / 4;                     // ... and per k-step
+    constexpr int XQ = BM == 256 ? 4 : 1, XW = BM == 256 ? 1 : AQ;      // rows (in eights) from copy to copy, wavefront to wavefront
     constexpr int SZW = 4 * 64 / GROUP;             // (scale, bias) words of four K-tiles
     constexpr int WL = 8 + (BLOCKS ? 2 * SZW : 2);  // weight + (scale, bias) loads per wavefront and four K-tiles
     constexpr int BLOCK_BYTES = 4 + GROUP / 2;      // blocks in place: one group
@@ -54,13 +54,18 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
     // tile of this workgroup: the workgroups of one XCD (id % 8) take consecutive tiles, row tiles of one column tile
     // first, so that they share that column tile's weights and a few row tiles' activations in the XCD's L2
     // (with K split over workgroups: all tiles of the first part of K, then those of the second ...)
-    const uint32_t tiles = a.tiles_m * a.tiles_n;
-    const uint32_t total = tiles * a.splits;
-    const uint32_t per_xcd = (total + 7) / 8;
-    const uint32_t t_id = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
-    if (t_id >= total) return;
+    // a last 256-row tile of at most 128 rows is short: the short tiles (of all column tiles and parts) come behind all
+    // others, so that they fill the gaps the whole tiles leave
+    const uint32_t rows_m = BM == 256 && a.short_rows ? a.tiles_m - 1 : a.tiles_m;     // row tiles of the first range
+    const uint32_t whole = rows_m * a.tiles_n, whole_total = whole * a.splits;
+    const uint32_t dealt = whole_total & ~7u;                             // dealt to the XCDs in runs; what is left follows
+    const uint32_t t_all = blockIdx.x < dealt ? (blockIdx.x % 8u) * (dealt / 8) + blockIdx.x / 8u : blockIdx.x;
+    if (t_all >= a.tiles_m * a.tiles_n * a.splits) return;
+    const bool is_short = BM == 256 && t_all >= whole_total;
+    const uint32_t t_id = is_short ? t_all - whole_total : t_all;
+    const uint32_t tiles = is_short ? a.tiles_n : whole;
     const uint32_t split = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t_id / tiles)), tile = t_id - split * tiles;
-    const uint32_t tn_all = tile / a.tiles_m, tm = tile % a.tiles_m;
+    const uint32_t tn_all = is_short ? tile : tile / rows_m, tm = is_short ? rows_m : tile % rows_m;
     // the matrix of this column tile (one of up to three that share the activations): its weights here, its result in
     // the epilogue, which asks again -- nothing of the choice is kept in registers over the K loop but the tile's number
     uint32_t tn = tn_all;
@@ -87,13 +92,14 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
     const uint32_t KT = (uint32_t)__builtin_amdgcn_readfirstlane((int)(kt_left < a.kt_per_split ? kt_left : a.kt_per_split));   // K-tiles of this workgroup: a multiple of four
 
     // ---- activations: global -> LDS ---------------------------------------------------------------
-    // copy q of wavefront w covers tile rows 8 (AQ w + q) .. + 7; lane L lands at row L / 8, position L % 8, and
+    // copy q of wavefront w covers tile rows 8 (4 q + w) .. + 7 of 256 (so that the first copies of all wavefronts are the
+    // rows a short tile needs), 8 (4 w + q) .. of 128 (the registers of that form are full: it spills the other way); lane L lands at row L / 8, position L % 8, and
     // fetches the chunk that belongs there after the rotation.  Rows past M re-read the last one.
     const uint32_t m_last = a.m - 1 - m0;           // last valid row of the tile
     uint32_t x_off[AQ];
 #pragma unroll
     for (int q = 0; q < AQ; q++) {
-        const uint32_t row = 8 * (AQ * wave + q) + (lane >> 3);
+        const uint32_t row = 8 * (XQ * q + XW * wave) + (lane >> 3);
         const uint32_t chunk = (lane & 7u) ^ ((row >> 1) & 7u);
         x_off[q] = (row < m_last ? row : m_last) * a.xs * 2 + chunk * 16;
     }
@@ -101,10 +107,10 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
     auto copy_x = [&](uint32_t kt, auto Q0, auto CNT) __attribute__((always_inline)) {
         const uint32_t t = kt < KT ? kt : KT - 1;   // past the end: a copy nobody reads, so that the counts stay the same
         const char* const g = wd_scalar(xg + (size_t)t * 128);
-        const uint32_t as = lds_base + (kt % kWideStages) * A_STAGE + wave * (AQ * 1024);
+        const uint32_t as = lds_base + (kt % kWideStages) * A_STAGE + wave * (XW * 1024);
 #pragma unroll
         for (int q = decltype(Q0)::value; q < decltype(Q0)::value + decltype(CNT)::value; q++) {
-            const uint32_t l = as + q * 1024;
+            const uint32_t l = as + q * (XQ * 1024);
             const uint32_t xo = x_off[q];
             asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(xo), "s"(g), "s"(l) : "memory");
         }
@@ -255,32 +261,36 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
     };
     // piece b of a word is the pair of codes (c0,c1) (c4,c5) (c2,c3) (c6,c7): its place among the operand's four registers
     auto dq_place = [](int b) constexpr { return ((b & 1) << 1) | (b >> 1); };
-    // One k-step = TM groups.  Group q: (every TM / CPK groups: one activation copy of K-tile kt_copy,) the read of
+    // One k-step = TM groups.  Group q: (one activation copy of K-tile kt_copy per four groups,) the read of
     // activation fragment q of the NEXT k-step (K-tile kt_next, word JN of K-tile TN of the current four), the two
     // MFMAs on fragment q of this one, and its share of the next k-step's weight fragments.
     u32x4 dq_o[2];
-    auto kstep = [&](auto BUF, auto TN, auto JN, uint32_t kt_next, uint32_t kt_copy, auto SLOT) __attribute__((always_inline)) {
+    auto kstep = [&](auto LIVE, auto BUF, auto TN, auto JN, uint32_t kt_next, uint32_t kt_copy, auto SLOT) __attribute__((always_inline)) {
         constexpr int buf = decltype(BUF)::value, tn_ = decltype(TN)::value, jn = decltype(JN)::value;
-        constexpr int slot = decltype(SLOT)::value;
+        constexpr int slot = decltype(SLOT)::value, live = decltype(LIVE)::value;     // activation fragments with rows below M
         const char* const xs_next = lds + (kt_next % kWideStages) * A_STAGE + a_rd[jn];
         const uint32_t tc = kt_copy < KT ? kt_copy : KT - 1;
         const char* const gx = wd_scalar(xg + (size_t)tc * 128);
-        const uint32_t lx = lds_base + (kt_copy % kWideStages) * A_STAGE + wave * (AQ * 1024);
+        const uint32_t lx = lds_base + (kt_copy % kWideStages) * A_STAGE + wave * (XW * 1024);
         static_for<TM>([&](auto Q) __attribute__((always_inline)) {
             constexpr int q = decltype(Q)::value;
-            if constexpr (q % (TM / CPK) == 0) {
-                constexpr int cq = slot * CPK + q / (TM / CPK);
-                const uint32_t l = lx + cq * 1024;
+            // copies of this slot (k-step): a quarter of the live ones each; with two live ones in slots 0 and 2
+            constexpr int cpk = live >= 4 ? live / 4 : 1;
+            if constexpr (q % (TM / cpk) == 0 && (live >= 4 || slot % 2 == 0)) {
+                constexpr int cq = live >= 4 ? slot * cpk + q / (TM / cpk) : slot / 2;
+                const uint32_t l = lx + cq * (XQ * 1024);
                 const uint32_t xo = x_off[cq];
                 asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(xo), "s"(gx), "s"(l) : "memory");
             }
-            xf[buf ^ 1][q] = *(const frag_t*)(xs_next + q * 4096);
-            if constexpr (XF16) {
-                acc[0][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[buf][0], xf[buf][q], acc[0][q], 0, 0, 0);
-                acc[1][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[buf][1], xf[buf][q], acc[1][q], 0, 0, 0);
-            } else {
-                acc[0][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][0], xf[buf][q], acc[0][q], 0, 0, 0);
-                acc[1][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][1], xf[buf][q], acc[1][q], 0, 0, 0);
+            if constexpr (q < live) {
+                xf[buf ^ 1][q] = *(const frag_t*)(xs_next + q * 4096);
+                if constexpr (XF16) {
+                    acc[0][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[buf][0], xf[buf][q], acc[0][q], 0, 0, 0);
+                    acc[1][q] = __builtin_amdgcn_mfma_f32_32x32x16_f16(wf[buf][1], xf[buf][q], acc[1][q], 0, 0, 0);
+                } else {
+                    acc[0][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][0], xf[buf][q], acc[0][q], 0, 0, 0);
+                    acc[1][q] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[buf][1], xf[buf][q], acc[1][q], 0, 0, 0);
+                }
             }
             // eight pieces (two fragments of four) over the TM groups
             static_for<8 / TM>([&](auto P) __attribute__((always_inline)) {
@@ -325,30 +335,43 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
     });
     __builtin_amdgcn_sched_barrier(0);
 
-    for (uint32_t kt0 = 0; kt0 < KT; kt0 += 4) {
-        static_for<4>([&](auto U) __attribute__((always_inline)) {
-            constexpr int u = decltype(U)::value;
-            const uint32_t kt = kt0 + u;
-            kstep(I0{}, U, I1{}, kt, kt + 2, I2{});
-            kstep(I1{}, U, I2{}, kt, kt + 2, I3{});
-            // K-tile kt + 1 has landed for everyone, K-tile kt - 1 is no longer read: its stage takes K-tile kt + 3.
-            // Younger than this wavefront's copies of K-tile kt + 1 are its copies of kt + 2 and, in iteration 1, the
-            // weight loads of iteration 0.
-            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(u == 1 ? AQ + WL : AQ) : "memory");
-            __builtin_amdgcn_s_barrier();
-            if constexpr (u == 0) load_w(kt0 / 4 + 1);
-            __builtin_amdgcn_sched_barrier(0);
-            kstep(I0{}, U, I3{}, kt, kt + 3, I0{});
-            if constexpr (u == 3) {
-                // the words of the next four K-tiles: younger are the copies of three K-tiles and those of k-step 2
-                take_w(std::integral_constant<int, 3 * AQ + CPK>{});
-                scales(I0{});
-                kstep(I1{}, I0{}, I0{}, kt + 1, kt + 3, I1{});
-            } else {
-                scales(std::integral_constant<int, u + 1>{});
-                kstep(I1{}, std::integral_constant<int, (u + 1) % 4>{}, I0{}, kt + 1, kt + 3, I1{});
-            }
-        });
+    auto walk = [&](auto LIVE) __attribute__((always_inline)) {
+        constexpr int live = decltype(LIVE)::value;     // = copies per wavefront and K-tile
+        for (uint32_t kt0 = 0; kt0 < KT; kt0 += 4) {
+            static_for<4>([&](auto U) __attribute__((always_inline)) {
+                constexpr int u = decltype(U)::value;
+                const uint32_t kt = kt0 + u;
+                kstep(LIVE, I0{}, U, I1{}, kt, kt + 2, I2{});
+                kstep(LIVE, I1{}, U, I2{}, kt, kt + 2, I3{});
+                // K-tile kt + 1 has landed for everyone, K-tile kt - 1 is no longer read: its stage takes K-tile kt + 3.
+                // Younger than this wavefront's copies of K-tile kt + 1 are its copies of kt + 2 and, in iteration 1, the
+                // weight loads of iteration 0.
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(u == 1 ? live + WL : live) : "memory");
+                __builtin_amdgcn_s_barrier();
+                if constexpr (u == 0) load_w(kt0 / 4 + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                kstep(LIVE, I0{}, U, I3{}, kt, kt + 3, I0{});
+                if constexpr (u == 3) {
+                    // the words of the next four K-tiles: younger are the copies of three K-tiles and those of k-step 2
+                    take_w(std::integral_constant<int, 3 * live + (live >= 4 ? live / 4 : 1)>{});
+                    scales(I0{});
+                    kstep(LIVE, I1{}, I0{}, I0{}, kt + 1, kt + 3, I1{});
+                } else {
+                    scales(std::integral_constant<int, u + 1>{});
+                    kstep(LIVE, I1{}, std::integral_constant<int, (u + 1) % 4>{}, I0{}, kt + 1, kt + 3, I1{});
+                }
+            });
+        }
+    };
+    // A short tile copies and multiplies a quarter or half of the fragments only (the accumulators of the others stay
+    // zero, their rows are past M).  The prologue has copied whole stages: a wait that counts fewer copies is then only
+    // stricter.
+    if constexpr (BM == 256) {
+        if (!is_short) walk(std::integral_constant<int, TM>{});
+        else if (m_last < 64) walk(std::integral_constant<int, 2>{});
+        else walk(std::integral_constant<int, 4>{});
+    } else {
+        walk(std::integral_constant<int, TM>{});
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (probing) {
@@ -550,6 +573,7 @@ template <int BM, bool SB_BF16, int GROUP, bool BLOCKS>
 mi355q_status launch_wide_tile(hipStream_t s, WideArgs a) {
     a.tiles_m = (a.m + BM - 1) / BM;
     if (a.segments <= 1) a.tiles_n = a.gated ? (a.n + kWideBN / 2 - 1) / (kWideBN / 2) : (a.n + kWideBN - 1) / kWideBN;
+    a.short_rows = wide_short_rows(a.m, BM) ? 1u : 0u;
     const uint32_t grid = (a.tiles_m * a.tiles_n * a.splits + 7) / 8 * 8;
     constexpr size_t lds = (size_t)kWideStages * BM * 128;
     auto kern = qgemm_wide_kernel<BM, SB_BF16, GROUP, BLOCKS, WIDE_XF16 != 0>;

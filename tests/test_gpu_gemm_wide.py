@@ -228,6 +228,32 @@ def test_wide_gemm_with_k_in_parts(pkg, ctx, tile_rows, parts):
         pkg.Context.probe_wide_shape(0, 0)
 
 
+@pytest.mark.parametrize("m", [257, 320, 321, 384, 385, 517])
+@pytest.mark.parametrize("parts", [1, 2])
+@pytest.mark.parametrize("f16", [False, True])
+def test_short_last_row_tile_of_256_rows_exact(pkg, ctx, m, parts, f16):
+    """A last 256-row tile of at most 64 or 128 rows copies and multiplies a part of its fragments only and comes behind
+    the whole tiles: edges of both, one row, one row more than is short; K in one and two parts, several column tiles
+    (so that the tiles are no multiple of eight).  Small integers: every result is exact."""
+    rng = np.random.default_rng(4700 + m + parts)
+    n, k = 3 * 256 + 12, 64 * 16 * parts + 256
+    codes = rng.integers(0, 16, (n, k), dtype=np.uint8)
+    scales = rng.choice([0.125, 0.25, 0.5], (n, k // 64))
+    zeros = rng.integers(-4, 5, (n, k // 64)) * 0.25
+    case = Case(4, 64, codes, scales, zeros)
+    x = rng.integers(-8, 9, (m, k)).astype(np.float32) * 0.125
+    want = x.astype(np.float64) @ (scales.repeat(64, axis=1) * codes + zeros.repeat(64, axis=1)).T
+    w = case.device_weight(ctx, pkg, pkg.LAYOUT_PLANES, pkg.BF16)
+    pkg.Context.probe_wide_shape(256, parts)
+    try:
+        say(f"short last tile m={m} parts={parts} f16={f16}")
+        got = run_qgemm(ctx, pkg, w, x, pkg.F32, wide(pkg), x_dtype=pkg.F16 if f16 else pkg.BF16)
+    finally:
+        pkg.Context.probe_wide_shape(0, 0)
+    assert np.array_equal(got.astype(np.float64), want)
+    w.destroy()
+
+
 @pytest.mark.parametrize("m", [128, 512, 2048])
 @pytest.mark.parametrize("n,k", [(14336, 4096), (4096, 14336)])
 def test_config3_prefill_as_dispatched(pkg, ctx, m, n, k):
