@@ -48,6 +48,7 @@ struct WView {
     uint32_t sz_stride;       // planes: 32-bit words from one row of sz to the next (>= blocks_per_row)
     uint32_t layout;          // mi355q_layout
     uint32_t sb_dtype;        // mi355q_dtype of scale/bias (F16 for STAF)
+    uint32_t far_scales;      // a bf16 scale of 2^104 or more among them
 };
 
 }  // namespace mi355q
@@ -107,6 +108,7 @@ struct mi355q_weight {
     // stream in memory.  Borrowed planes (wrap) keep the caller's codes and an owned sz plane.
     uint32_t code_stride, sz_stride;   // in 32-bit words
     uint8_t sz_separate;               // sz is an allocation of its own (borrowed planes)
+    uint8_t far_scales;                // borrowed bf16 planes: a scale of 2^104 or more (or no number) was met packing sz
     size_t blocks_bytes, codes_bytes, sb_bytes;
     mi355q::WView view() const {
         mi355q::WView v;
@@ -127,6 +129,7 @@ struct mi355q_weight {
         v.sz_stride = sz_stride;
         v.layout = layout;
         v.sb_dtype = sb_dtype;
+        v.far_scales = far_scales;
         return v;
     }
 };
@@ -169,8 +172,9 @@ mi355q_status launch_argmax_finish(hipStream_t s, const unsigned long long* part
 constexpr uint32_t kArgmaxStandaloneKeys = 256;
 mi355q_status launch_argmax(hipStream_t s, const void* logits, int dtype, uint32_t n,
                             int32_t* token_out, unsigned long long* partial);
+// (`far`: null, or a zeroed word that becomes 1 if a scale, read as bf16, is 2^104 or more, infinite or no number)
 mi355q_status launch_pack_sz(hipStream_t s, const uint16_t* scales, const uint16_t* biases, uint32_t* sz,
-                             size_t groups, uint32_t blocks_per_row, uint32_t sz_stride);
+                             size_t groups, uint32_t blocks_per_row, uint32_t sz_stride, uint32_t* far);
 
 // Fast split-plane GEMV (kernels_gemv.hip).  can_* say whether a shape is eligible.
 bool gemv_fast_eligible(const WView& w, int x_dtype, uint32_t m, uint32_t x_stride);

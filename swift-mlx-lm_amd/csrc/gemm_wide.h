@@ -49,8 +49,15 @@ constexpr int kWideBN = 256;
 // the fragments and are dispatched behind all others.
 inline bool wide_short_rows(uint32_t m, uint32_t bm) { return bm == 256 && m > bm && m % bm != 0 && m % bm <= 128; }
 
+// Type of a weight's scales and zeros as the kernel reads them: f16; bf16 below 2^104 (every prepared weight: the values
+// an f16 header would hold), which times 2^24 stays finite; any bf16 (borrowed planes with a scale beyond that).
+enum : uint32_t { kWideScalesF16 = 0, kWideScalesBf16 = 1, kWideScalesBf16Any = 2 };
+inline uint32_t wide_scales(const WView& w) {
+    return w.sb_dtype != MI355Q_BF16 ? kWideScalesF16 : w.far_scales ? kWideScalesBf16Any : kWideScalesBf16;
+}
+
 // the kernel launch alone (tiles_m, tiles_n filled in here); activations bf16 / f16
-mi355q_status launch_wide_kernel_bf16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, bool sb_bf16, bool blocks);
-mi355q_status launch_wide_kernel_f16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, bool sb_bf16, bool blocks);
+mi355q_status launch_wide_kernel_bf16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, uint32_t scales, bool blocks);
+mi355q_status launch_wide_kernel_f16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, uint32_t scales, bool blocks);
 
 }  // namespace mi355q

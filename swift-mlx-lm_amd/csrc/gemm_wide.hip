@@ -245,9 +245,8 @@ mi355q_status launch_qgemm_wide(hipStream_t s, mi355q_context* ctx, const WView&
         if (mi355q_status st = ensure_workspace(ctx, part_bytes)) return st;
         a.partial = (float*)ctx->workspace;
     }
-    const bool sb_bf16 = w.sb_dtype == MI355Q_BF16;
-    if (mi355q_status st = x_dtype == MI355Q_F16 ? launch_wide_kernel_f16(s, a, g.bm, w.group, sb_bf16, blocks)
-                                                 : launch_wide_kernel_bf16(s, a, g.bm, w.group, sb_bf16, blocks))
+    if (mi355q_status st = x_dtype == MI355Q_F16 ? launch_wide_kernel_f16(s, a, g.bm, w.group, wide_scales(w), blocks)
+                                                 : launch_wide_kernel_bf16(s, a, g.bm, w.group, wide_scales(w), blocks))
         return st;
     if (a.partial) {
         size_t wgs = ((size_t)a.m * a.n / 4 + 255) / 256;
@@ -377,9 +376,10 @@ mi355q_status launch_qgemm_wide_multi(hipStream_t s, mi355q_context* ctx, uint32
         if (mi355q_status st = ensure_workspace(ctx, (size_t)g.splits * m * cols * sizeof(float))) return st;
         a.partial = (float*)ctx->workspace;
     }
-    const bool sb_bf16 = w[0].sb_dtype == MI355Q_BF16;
-    if (mi355q_status st = x_dtype == MI355Q_F16 ? launch_wide_kernel_f16(s, a, g.bm, w[0].group, sb_bf16, blocks)
-                                                 : launch_wide_kernel_bf16(s, a, g.bm, w[0].group, sb_bf16, blocks))
+    uint32_t scales = 0;                               // one form for all: the widest any of them asks for
+    for (uint32_t i = 0; i < count; i++) scales = wide_scales(w[i]) > scales ? wide_scales(w[i]) : scales;
+    if (mi355q_status st = x_dtype == MI355Q_F16 ? launch_wide_kernel_f16(s, a, g.bm, w[0].group, scales, blocks)
+                                                 : launch_wide_kernel_bf16(s, a, g.bm, w[0].group, scales, blocks))
         return st;
     if (a.partial) {
         sum.partial = a.partial; sum.m = m; sum.n_total = cols; sum.splits = g.splits; sum.y_dtype = (uint32_t)y_dtype;
@@ -447,9 +447,9 @@ mi355q_status launch_qgemm_wide_gated(hipStream_t s, mi355q_context* ctx, const 
     a.y_dtype = (uint32_t)y_dtype;
     a.line_stores = ((size_t)y_stride * (y_dtype == MI355Q_F32 ? 4 : 2) % 16 == 0 && (uintptr_t)y % 16 == 0) ? 1u : 0u;
     a.splits = 1; a.kt_per_split = gate.k / 64;
-    const bool sb_bf16 = gate.sb_dtype == MI355Q_BF16;
-    return x_dtype == MI355Q_F16 ? launch_wide_kernel_f16(s, a, g.bm, gate.group, sb_bf16, blocks)
-                                 : launch_wide_kernel_bf16(s, a, g.bm, gate.group, sb_bf16, blocks);
+    const uint32_t scales = wide_scales(gate) > wide_scales(up) ? wide_scales(gate) : wide_scales(up);
+    return x_dtype == MI355Q_F16 ? launch_wide_kernel_f16(s, a, g.bm, gate.group, scales, blocks)
+                                 : launch_wide_kernel_bf16(s, a, g.bm, gate.group, scales, blocks);
 }
 
 }  // namespace mi355q

@@ -36,7 +36,8 @@ __device__ __forceinline__ const char* wd_scalar(const char* p) {
 // BLOCKS: the weights are the reference's interleaved blocks read in place (f16 scale, f16 zero, then the group's codes:
 // 36 bytes per 64 codes, 68 per 128); a lane's sixteen code bytes then sit at a 4-byte aligned address and the
 // (scale, zero) pair of a K-tile is one more 4-byte load.  XF16: f16 activations, weights rounded to f16, f16 MFMA.
-template <int BM, bool SB_BF16, int GROUP, bool BLOCKS, bool XF16>
+// SCALES (kWideScales*): the type of the scales and zeros, and for bf16 whether they may be out of reach of the f16 form.
+template <int BM, int SCALES, int GROUP, bool BLOCKS, bool XF16>
 __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(WideArgs a) {
     constexpr int TM = BM / 32;                     // activation fragments = groups per k-step
     constexpr int A_STAGE = BM * 128;
@@ -232,26 +233,41 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
 #pragma unroll
         for (int f = 0; f < 2; f++) {
             const uint32_t szw = szcur[f][t * 64 / GROUP];
-            if constexpr (SB_BF16) {
+            if constexpr (SCALES != kWideScalesF16) {
                 sc[f] = __uint_as_float(szw << 16); zr[f] = __uint_as_float(szw & 0xFFFF0000u);
             } else {
                 sc[f] = f16_to_f32((uint16_t)(szw & 0xFFFFu)); zr[f] = f16_to_f32((uint16_t)(szw >> 16));
             }
-            // the codes' fields as f16 numbers (dq_piece) are q * 2^-24 and, one nibble up, q * 2^-20
-            sc16[f] = sc[f] * 0x1p20f;
-            sc[f] *= 0x1p24f;
+            if constexpr (SCALES == kWideScalesBf16Any) {
+                sc16[f] = sc[f] * 0.0625f;          // exact: bf16 subnormals keep their bits four binades down in fp32
+            } else {
+                // the codes' fields as f16 numbers (dq_piece) are q * 2^-24 and, one nibble up, q * 2^-20
+                sc16[f] = sc[f] * 0x1p20f;
+                sc[f] *= 0x1p24f;
+            }
         }
     };
     // a quarter of the dequantisation of word w of fragment f: codes 2 p and 2 p + 1 as one packed pair of the
     // activations' type.  The pieces come in the order p = 0, 2, 1, 3.  A nibble alone in the low seven bits' reach of a
     // half-word is, read as f16, the (subnormal) number q * 2^-24, or q * 2^-20 a nibble further up, and the mixed-type
     // fma takes either half of a register as such a number: fma(scale * 2^24, q * 2^-24, bias) is fma(scale, q, bias) bit
-    // for bit (powers of two; a bf16 scale would have to reach 2^104 to leave the range), with no conversion, where byte
-    // extraction plus convert took 22 instructions for eight codes and this takes 17 (a Llama-3-8B layer's projections at
-    // 128 / 2048 bf16 rows 168.5 -> 165.3 / 813 -> 800 us, at 517 fp32 rows 659 -> 643; same bits).
+    // for bit (powers of two), with no conversion, where byte extraction plus convert took 22 instructions for eight codes
+    // and this takes 17 (a Llama-3-8B layer's projections at 128 / 2048 bf16 rows 168.5 -> 165.3 / 813 -> 800 us, at 517
+    // fp32 rows 659 -> 643; same bits).  A bf16 scale of 2^104 or more would leave the fp32 range times 2^24 (and give
+    // infinity times code 0): weights that hold one (kWideScalesBf16Any; only borrowed planes can) have their bytes converted.
+    // piece b of a word is the pair of codes (c0,c1) (c4,c5) (c2,c3) (c6,c7): its place among the operand's four registers
+    auto dq_place = [](int b) constexpr { return ((b & 1) << 1) | (b >> 1); };
     uint32_t dq_t[2], dq_u[2];
     auto dq_piece = [&](auto F, auto B, uint32_t w) __attribute__((always_inline)) -> uint32_t {
         constexpr int f = decltype(F)::value, b = decltype(B)::value;
+        if constexpr (SCALES == kWideScalesBf16Any) {
+            // codes 2 p and 2 p + 1: byte p of the even and of the odd nibbles, which stay sixteen times too large
+            constexpr int p = dq_place(b);
+            if constexpr (b == 0) { dq_t[f] = w & 0x0F0F0F0Fu; dq_u[f] = w & 0xF0F0F0F0u; }
+            const float v0 = __builtin_fmaf((float)((dq_t[f] >> (8 * p)) & 0xFFu), sc[f], zr[f]);
+            const float v1 = __builtin_fmaf((float)((dq_u[f] >> (8 * p)) & 0xFFu), sc16[f], zr[f]);
+            return XF16 ? wd_pack_f16(v0, v1) : wd_pack_bf16(v0, v1);
+        }
         constexpr int half = b & 1;
         if constexpr (b == 0) { dq_t[f] = w & 0x000F000Fu; dq_u[f] = w & 0x00F000F0u; }                   // c0 c4, c1 c5
         if constexpr (b == 2) { dq_t[f] = (w >> 8) & 0x000F000Fu; dq_u[f] = (w >> 8) & 0x00F000F0u; }     // c2 c6, c3 c7
@@ -259,8 +275,6 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
         const float w1 = __builtin_fmaf((float)__builtin_bit_cast(wd_f16x2_v, dq_u[f])[half], sc16[f], zr[f]);
         return XF16 ? wd_pack_f16(w0, w1) : wd_pack_bf16(w0, w1);
     };
-    // piece b of a word is the pair of codes (c0,c1) (c4,c5) (c2,c3) (c6,c7): its place among the operand's four registers
-    auto dq_place = [](int b) constexpr { return ((b & 1) << 1) | (b >> 1); };
     // One k-step = TM groups.  Group q: (one activation copy of K-tile kt_copy per four groups,) the read of
     // activation fragment q of the NEXT k-step (K-tile kt_next, word JN of K-tile TN of the current four), the two
     // MFMAs on fragment q of this one, and its share of the next k-step's weight fragments.
@@ -569,35 +583,42 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
 }
 
 
-template <int BM, bool SB_BF16, int GROUP, bool BLOCKS>
+template <int BM, int SCALES, int GROUP, bool BLOCKS>
 mi355q_status launch_wide_tile(hipStream_t s, WideArgs a) {
     a.tiles_m = (a.m + BM - 1) / BM;
     if (a.segments <= 1) a.tiles_n = a.gated ? (a.n + kWideBN / 2 - 1) / (kWideBN / 2) : (a.n + kWideBN - 1) / kWideBN;
     a.short_rows = wide_short_rows(a.m, BM) ? 1u : 0u;
     const uint32_t grid = (a.tiles_m * a.tiles_n * a.splits + 7) / 8 * 8;
     constexpr size_t lds = (size_t)kWideStages * BM * 128;
-    auto kern = qgemm_wide_kernel<BM, SB_BF16, GROUP, BLOCKS, WIDE_XF16 != 0>;
+    auto kern = qgemm_wide_kernel<BM, SCALES, GROUP, BLOCKS, WIDE_XF16 != 0>;
     if (mi355q_status st = raise_lds_limit((const void*)kern, lds)) return st;
     kern<<<dim3(grid), dim3(256), lds, s>>>(a);
     MI355Q_HIP(hipGetLastError());
     return MI355Q_OK;
 }
 
+template <int BM, int SCALES>
+mi355q_status launch_wide_planes(hipStream_t s, const WideArgs& a, uint32_t group) {
+    return group == 64 ? launch_wide_tile<BM, SCALES, 64, false>(s, a) : launch_wide_tile<BM, SCALES, 128, false>(s, a);
+}
+
 template <int BM>
-mi355q_status launch_wide_bm(hipStream_t s, const WideArgs& a, uint32_t group, bool sb_bf16, bool blocks) {
-    if (blocks) return group == 64 ? launch_wide_tile<BM, false, 64, true>(s, a) : launch_wide_tile<BM, false, 128, true>(s, a);
-    if (group == 64) return sb_bf16 ? launch_wide_tile<BM, true, 64, false>(s, a) : launch_wide_tile<BM, false, 64, false>(s, a);
-    return sb_bf16 ? launch_wide_tile<BM, true, 128, false>(s, a) : launch_wide_tile<BM, false, 128, false>(s, a);
+mi355q_status launch_wide_bm(hipStream_t s, const WideArgs& a, uint32_t group, uint32_t scales, bool blocks) {
+    if (blocks)
+        return group == 64 ? launch_wide_tile<BM, kWideScalesF16, 64, true>(s, a) : launch_wide_tile<BM, kWideScalesF16, 128, true>(s, a);
+    if (scales == kWideScalesF16) return launch_wide_planes<BM, kWideScalesF16>(s, a, group);
+    if (scales == kWideScalesBf16) return launch_wide_planes<BM, kWideScalesBf16>(s, a, group);
+    return launch_wide_planes<BM, kWideScalesBf16Any>(s, a, group);
 }
 
 }  // namespace
 
 #if WIDE_XF16
-mi355q_status launch_wide_kernel_f16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, bool sb_bf16, bool blocks) {
+mi355q_status launch_wide_kernel_f16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, uint32_t scales, bool blocks) {
 #else
-mi355q_status launch_wide_kernel_bf16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, bool sb_bf16, bool blocks) {
+mi355q_status launch_wide_kernel_bf16(hipStream_t s, WideArgs a, uint32_t bm, uint32_t group, uint32_t scales, bool blocks) {
 #endif
-    return bm == 256 ? launch_wide_bm<256>(s, a, group, sb_bf16, blocks) : launch_wide_bm<128>(s, a, group, sb_bf16, blocks);
+    return bm == 256 ? launch_wide_bm<256>(s, a, group, scales, blocks) : launch_wide_bm<128>(s, a, group, scales, blocks);
 }
 
 }  // namespace mi355q

@@ -37,21 +37,24 @@ mi355q_status launch_unpack_codes(hipStream_t s, const WView& w, uint8_t* out) {
 __global__ __launch_bounds__(256) void pack_sz_kernel(const uint16_t* __restrict__ scales,
                                                       const uint16_t* __restrict__ biases,
                                                       uint32_t* __restrict__ sz, size_t groups,
-                                                      uint32_t blocks_per_row, uint32_t sz_stride) {
+                                                      uint32_t blocks_per_row, uint32_t sz_stride,
+                                                      uint32_t* __restrict__ far) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     const size_t stride = (size_t)gridDim.x * blockDim.x;
     for (; i < groups; i += stride) {
         const size_t row = i / blocks_per_row, b = i - row * blocks_per_row;
-        sz[row * sz_stride + b] = (uint32_t)scales[i] | ((uint32_t)biases[i] << 16);
+        const uint32_t scale = scales[i];
+        sz[row * sz_stride + b] = scale | ((uint32_t)biases[i] << 16);
+        if (far && (scale & 0x7FFFu) >= 0x7380u) *far = 1;               // bf16 exponent field of 2^104: 231
     }
 }
 
 mi355q_status launch_pack_sz(hipStream_t s, const uint16_t* scales, const uint16_t* biases, uint32_t* sz,
-                             size_t groups, uint32_t blocks_per_row, uint32_t sz_stride) {
+                             size_t groups, uint32_t blocks_per_row, uint32_t sz_stride, uint32_t* far) {
     size_t blocks = (groups + 255) / 256;
     if (blocks > 8192) blocks = 8192;
     if (blocks == 0) blocks = 1;
-    pack_sz_kernel<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(scales, biases, sz, groups, blocks_per_row, sz_stride);
+    pack_sz_kernel<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(scales, biases, sz, groups, blocks_per_row, sz_stride, far);
     MI355Q_HIP(hipGetLastError());
     return MI355Q_OK;
 }

@@ -231,11 +231,11 @@ mi355q_status upload_new(void** dev, const void* host, size_t bytes) {
 
 // Packed (scale, bias) words of a split-plane weight, filled once on the device from the two
 // 16-bit planes.  `dst` is either the sz part of the row-interleaved buffer or a plane of its own.
-mi355q_status fill_sz(mi355q_weight* w) {
+mi355q_status fill_sz(mi355q_weight* w, uint32_t* far = nullptr) {
     const uint32_t bpr = (uint32_t)(w->k / w->fmt.group_size);
     const size_t groups = (size_t)w->n * bpr;
     if (mi355q_status st = launch_pack_sz(nullptr, (const uint16_t*)w->scales, (const uint16_t*)w->biases,
-                                          (uint32_t*)w->sz, groups, bpr, w->sz_stride))
+                                          (uint32_t*)w->sz, groups, bpr, w->sz_stride, far))
         return st;
     MI355Q_HIP(hipStreamSynchronize(nullptr));
     return MI355Q_OK;
@@ -247,8 +247,17 @@ mi355q_status build_sz_plane(mi355q_weight* w) {
     w->code_stride = (uint32_t)(w->k * w->fmt.bits / 32);
     w->sz_stride = bpr;
     w->sz_separate = 1;
-    MI355Q_HIP(hipMalloc(&w->sz, (size_t)w->n * bpr * 4));
-    return fill_sz(w);
+    const size_t words = (size_t)w->n * bpr;
+    MI355Q_HIP(hipMalloc(&w->sz, (words + 1) * 4));
+    if (w->sb_dtype != MI355Q_BF16) return fill_sz(w);
+    // the caller's bf16 scales may be any number (those prepared here went through f16): the word behind sz says so
+    uint32_t* const far = (uint32_t*)w->sz + words;
+    uint32_t met = 0;
+    MI355Q_HIP(hipMemset(far, 0, 4));
+    if (mi355q_status st = fill_sz(w, far)) return st;
+    MI355Q_HIP(hipMemcpy(&met, far, 4, hipMemcpyDeviceToHost));
+    w->far_scales = met != 0;
+    return MI355Q_OK;
 }
 
 // Owned planes: one buffer of rows [code words | sz words | pad to 16 bytes].  The host code plane

@@ -254,6 +254,84 @@ def test_short_last_row_tile_of_256_rows_exact(pkg, ctx, m, parts, f16):
     w.destroy()
 
 
+def _wrapped(pkg, ctx, group, codes, scales, zeros):
+    """Borrowed bf16 planes (mi355q_weight_wrap_planes): the only weights whose scales may be any bf16 number."""
+    n, k = codes.shape
+    fmt = pkg.QuantizationFormatRegistry.format_for_mlx_quantization(4, group)
+    bufs = [ctx.upload(kat.mlx_planes(codes, 4)), ctx.upload(oracle.bf16_from_f32(scales.astype(np.float32))),
+            ctx.upload(oracle.bf16_from_f32(zeros.astype(np.float32)))]
+    return ctx.weight_wrap_planes(fmt, n, k, *bufs, pkg.BF16), bufs
+
+
+@pytest.mark.parametrize("group,tile_rows", [(64, 256), (64, 128), (128, 256), (128, 128)])
+@pytest.mark.parametrize("x_name", ["BF16", "F32", "F16"])
+def test_borrowed_bf16_scales_beyond_2_to_the_104(pkg, ctx, group, tile_rows, x_name):
+    """bf16 scales whose product with 2^24 is no fp32 number any more, beside ordinary ones: finite, and exact.  Units of
+    2^108 (weights of at most eight bits) against activations in units of 2^-110 keep every sum an integer multiple of
+    2^-2 below 2^17.  f16 activations (whose weights are rounded to f16) meet code 0 alone: the zero point."""
+    rng = np.random.default_rng(4900 + group + tile_rows)
+    f16 = x_name == "F16"
+    m, n, k = 300, 264, 2 * 256                          # a 256-row tile and a short one; three 128-row tiles
+    codes = np.zeros((n, k), np.uint8) if f16 else rng.integers(0, 16, (n, k), dtype=np.uint8)
+    scales = rng.choice([1.0, 2.0, 4.0], (n, k // group)) * (2.0 ** 108)
+    if f16:
+        scales[::3] = 0.25
+    zeros = rng.integers(-4, 5, (n, k // group)) * (0.25 if f16 else 2.0 ** 108)
+    x = (rng.integers(-8, 9, (m, k)) * (0.125 if f16 else 2.0 ** -110)).astype(np.float32)
+    want = x.astype(np.float64) @ (scales.repeat(group, axis=1) * codes + zeros.repeat(group, axis=1)).T
+    w, bufs = _wrapped(pkg, ctx, group, codes, scales, zeros)
+    pkg.Context.probe_wide_shape(tile_rows, 1)
+    try:
+        say(f"scales beyond 2^104 g{group} tile {tile_rows} x={x_name}")
+        got = run_qgemm(ctx, pkg, w, x, pkg.F32, wide(pkg), x_dtype=getattr(pkg, x_name))
+    finally:
+        pkg.Context.probe_wide_shape(0, 0)
+    assert np.array_equal(got.astype(np.float64), want)
+    w.destroy()
+    for b in bufs:
+        b.free()
+
+
+def test_borrowed_bf16_scales_beyond_2_to_the_104_in_shared_and_gated_launches(pkg, ctx):
+    """One such matrix beside an ordinary one in a shared launch and in a gated pair: both are exact."""
+    rng = np.random.default_rng(4950)
+    m, n, k = 130, 256, 2 * 256
+    codes = [rng.integers(0, 16, (n, k), dtype=np.uint8) for _ in range(2)]
+    unit = [2.0 ** 108, 2.0 ** 100]
+    scales = [rng.choice([1.0, 2.0, 4.0], (n, k // 64)) * u for u in unit]
+    zeros = [rng.integers(-4, 5, (n, k // 64)) * u for u in unit]
+    x = (rng.integers(-8, 9, (m, k)) * 2.0 ** -110).astype(np.float32)
+    want = [x.astype(np.float64) @ (s.repeat(64, axis=1) * c + z.repeat(64, axis=1)).T for c, s, z in zip(codes, scales, zeros)]
+    made = [_wrapped(pkg, ctx, 64, c, s, z) for c, s, z in zip(codes, scales, zeros)]
+    ws = [w for w, _ in made]
+    xdev = ctx.upload(oracle.bf16_from_f32(x))
+    for order in ((0, 1), (1, 0)):
+        outs = [ctx.alloc(m * n * 4) for _ in order]
+        say("scales beyond 2^104, shared launch, order", order)
+        ctx.batched_qgemm([ws[i] for i in order], xdev, pkg.BF16, outs, pkg.F32, m, flags=pkg.FLAG_PROBE_WIDE)
+        ctx.synchronize()
+        for i, o in zip(order, outs):
+            assert np.array_equal(o.download(np.float32, (m, n)).astype(np.float64), want[i]), (order, i)
+            o.free()
+        y = ctx.alloc(m * n * 4)
+        say("scales beyond 2^104, gated launch, order", order)
+        ctx.gated_qgemm(ws[order[0]], ws[order[1]], xdev, pkg.BF16, y, pkg.F32, m, flags=pkg.FLAG_PROBE_WIDE)
+        ctx.synchronize()
+        gate, up = (want[i] for i in order)
+        with np.errstate(over="ignore"):
+            silu = gate / (1.0 + np.exp(-gate)) * up
+        got = y.download(np.float32, (m, n)).astype(np.float64)
+        # the activation's own 4e-7 and the roundings of the products, and e^-gate of a gate rounded times log2(e): 2^-24 of
+        # the exponent, doubled; 1e-30: where fp32 ends
+        assert np.all(np.abs(got - silu) <= (2e-6 + 2.0 ** -23 * np.abs(np.minimum(gate, 0))) * np.abs(silu) + 1e-30)
+        y.free()
+    xdev.free()
+    for w, bufs in made:
+        w.destroy()
+        for b in bufs:
+            b.free()
+
+
 @pytest.mark.parametrize("m", [128, 512, 2048])
 @pytest.mark.parametrize("n,k", [(14336, 4096), (4096, 14336)])
 def test_config3_prefill_as_dispatched(pkg, ctx, m, n, k):
