@@ -388,12 +388,18 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
         walk(std::integral_constant<int, TM>{});
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // the lane's number counted again: what the epilogue derives from it is then not shared with the offsets of the loads
+    // above and kept over the K loop, in registers that the 128-row form does not have (it spilled up to two for them)
+    uint32_t all_lanes = ~0u;
+    asm volatile("" : "+s"(all_lanes));
+    const uint32_t lane_e = __builtin_amdgcn_mbcnt_hi(all_lanes, __builtin_amdgcn_mbcnt_lo(all_lanes, 0));
     if (probing) {
         const unsigned long long c1 = __builtin_readcyclecounter(), r1 = __builtin_amdgcn_s_memrealtime();
-        if (lane == 0) { a.probe[0] = c1 - probe_c0; a.probe[1] = r1 - probe_r0; }
+        if (lane_e == 0) { a.probe[0] = c1 - probe_c0; a.probe[1] = r1 - probe_r0; }
     }
 
     // ---- epilogue: one rounding, to the output type -----------------------------------------------------
+    const uint32_t ln_e = lane_e & 31, lh_e = lane_e >> 5;
     // the result of this tile's matrix (asked again, from a copy of the tile's number the compiler takes for another)
     uint32_t tn_again = tn_all;
     asm volatile("" : "+s"(tn_again));
@@ -413,14 +419,14 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
         static_for<2>([&](auto F) __attribute__((always_inline)) {
             static_for<TM>([&](auto I) __attribute__((always_inline)) {
                 constexpr int f = decltype(F)::value, i = decltype(I)::value;
-                const uint32_t row = m0 + i * 32 + ln;
+                const uint32_t row = m0 + i * 32 + ln_e;
                 // an opaque touch per output type: identical register fetches in the three copies of this loop would
                 // otherwise be merged in front of the branch, all 256 at once
                 asm volatile("" : "+v"(acc[f][i]));
                 if (row < a.m) {
 #pragma unroll
                     for (int g = 0; g < 4; g++) {
-                        const uint32_t col = n0 + 64 * wave + 32 * f + 8 * g + 4 * lh;
+                        const uint32_t col = n0 + 64 * wave + 32 * f + 8 * g + 4 * lh_e;
                         const float v[4] = {acc[f][i][4 * g + 0], acc[f][i][4 * g + 1], acc[f][i][4 * g + 2], acc[f][i][4 * g + 3]};
                         const size_t o = (size_t)row * ys + col;
                         if (wide && col + 3 < seg_n) {
@@ -469,7 +475,7 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
                     const float v0 = acc[f][i][4 * g + 0], v1 = acc[f][i][4 * g + 1], v2 = acc[f][i][4 * g + 2], v3 = acc[f][i][4 * g + 3];
-                    char* const at = stage + ln * PITCH + (32 * f + 8 * g + 4 * lh) * ESZ;
+                    char* const at = stage + ln_e * PITCH + (32 * f + 8 * g + 4 * lh_e) * ESZ;
                     if constexpr (dt == MI355Q_F32) {
                         const wd_float4_v t = {v0, v1, v2, v3};
                         *(wd_float4_v*)at = t;
@@ -485,7 +491,7 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
             for (int t = 0; t < 32 / RPI; t++) {
-                const uint32_t r = t * RPI + lane / LPR, piece = lane % LPR;
+                const uint32_t r = t * RPI + lane_e / LPR, piece = lane_e % LPR;
                 const u32x4 d = *(const u32x4*)(stage + r * PITCH + piece * 16);
                 const uint32_t row = m0 + i * 32 + r;
                 if (row < a.m)
@@ -518,7 +524,7 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
             if (whole) {
 #pragma unroll
                 for (int g = 0; g < 4; g++) {
-                    char* const at = stage + ln * PITCH + (8 * g + 4 * lh) * ESZ;
+                    char* const at = stage + ln_e * PITCH + (8 * g + 4 * lh_e) * ESZ;
                     if constexpr (dt == MI355Q_F32) {
                         const wd_float4_v t = {v[4 * g], v[4 * g + 1], v[4 * g + 2], v[4 * g + 3]};
                         *(wd_float4_v*)at = t;
@@ -534,7 +540,7 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
                 for (int t = 0; t < 32 / RPI; t++) {
-                    const uint32_t r = t * RPI + lane / LPR, piece = lane % LPR;
+                    const uint32_t r = t * RPI + lane_e / LPR, piece = lane_e % LPR;
                     const u32x4 d = *(const u32x4*)(stage + r * PITCH + piece * 16);
                     const uint32_t row = m0 + i * 32 + r;
                     if (row < a.m)
@@ -544,11 +550,11 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
                 __builtin_amdgcn_wave_barrier();
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             } else {
-                const uint32_t row = m0 + i * 32 + ln;
+                const uint32_t row = m0 + i * 32 + ln_e;
                 if (row < a.m) {
 #pragma unroll
                     for (int r = 0; r < 16; r++) {
-                        const uint32_t col = n0 + 32 * wave + 8 * (r / 4) + 4 * lh + r % 4;
+                        const uint32_t col = n0 + 32 * wave + 8 * (r / 4) + 4 * lh_e + r % 4;
                         if (col < seg_n) store_out<dt>(seg_y, (size_t)row * seg_ys + col, v[r]);
                     }
                 }

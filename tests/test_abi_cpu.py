@@ -2,6 +2,7 @@
 host-only entry points (format registry, MLX->STAF repack, shape families, error paths) behave
 like the reference interface they replace.  No compute entry point is called here."""
 import ctypes as C
+import struct
 import subprocess
 
 import numpy as np
@@ -25,6 +26,25 @@ def test_library_loads_and_exports_every_declared_symbol():
     for name in names:
         assert name in exported, name
         getattr(lib, name)
+
+
+def test_no_instantiation_of_the_wide_tile_kernel_spills():
+    """The wide-tile prefill kernel loads its weights with hand-written instructions whose data arrives after the statement
+    that issued them, so none of its instantiations may spill a vector register: read from the metadata notes of the
+    library's own code objects (two activation types x two tile heights x planes and blocks x two groups x scale types)."""
+    msgpack = pytest.importorskip("msgpack")
+    with open(pkg.LIB_PATH, "rb") as f:
+        image = f.read()
+    spills, at = {}, image.find(b"AMDGPU\0\0")
+    while at >= 0:
+        name_size, size, kind = struct.unpack("<III", image[at - 12:at])
+        if (name_size, kind) == (7, 32):
+            notes = msgpack.unpackb(image[at + 8:at + 8 + size], raw=False, strict_map_key=False)
+            spills.update({k[".name"]: k[".vgpr_spill_count"] for k in notes.get("amdhsa.kernels", [])})
+        at = image.find(b"AMDGPU\0\0", at + 8)
+    wide = {k: n for k, n in spills.items() if "qgemm_wide_kernel" in k}
+    assert len(wide) == 2 * 2 * (3 * 2 + 2), sorted(wide)
+    assert not any(wide.values()), {k: n for k, n in wide.items() if n}
 
 
 # ---- T/SupportedQuantizationsContractTests.swift: registry <-> documented table ------------
