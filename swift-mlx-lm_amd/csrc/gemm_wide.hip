@@ -126,11 +126,17 @@ void gemm_wide_force_shape(uint32_t bm, uint32_t splits) {
     g_wide_forced_splits.store(splits <= 8 ? splits : 0, std::memory_order_relaxed);
 }
 
-// Cycles per K-tile of a short tile (256-row form, at most 64 or 128 rows of it used).  Measured: 1300 to 1450 at 5 rows
-// (gate+up 4096 -> 2 x 14336 at 517 rows against 512: 160 against 108 us, fp32 297 against 204; the weights are dequantised
-// all the same).  Carried higher, because the cost of K parts below is low for wide results: with 1000 to 1600 that pair at
-// 270 fp32 rows went to two parts, 184 us against 169 in one, and q+k+v at 517 to four, 90 against 82 in two of 128 rows.
-constexpr double kWideShort64 = 1800.0, kWideShort128 = 1900.0;
+// What the choice below charges for short tiles (256-row form, at most 64 or 128 rows of it used) that take rounds of their
+// own: cycles per K-tile, the 8 us of any round, and a share of the whole cost where K is in parts.  Fitted, not the cycles
+// of one tile (those are 1000 to 1150 and 1400 to 1550, from 4096 and 8192 -> 28672 at 512, 517 and 640 rows: 107 / 151 /
+// 165 and 208 / 299 / 330 us).  They stand in for what the model leaves out: whole tiles that leave CUs idle run at a higher
+// clock than the 2500 cycles below assume (8192 -> 28672 at 270 rows in one part 171 us, charged 191), so splitting K looks
+// better than it is.  Against 186 problems measured at every tile height and number of parts (4096 to 65536 columns, K walks
+// of 4096 to 28672, 128 to 2432 rows) the choice is nowhere more than 1.5 % slower than it was without short tiles, and
+// within 4 % of the fastest shape in all but nine (worst 10 %).  With 1800 / 1900 cycles alone, neither the round's 8 us nor
+// the share, 22 of them went into K parts that were slower than before (8192 -> 16384 at 320 rows 116 us in four parts
+// against 107 in two; 11008 -> 24576 at 384 rows 235 in four against 213 in one).
+constexpr double kWideShort64 = 1800.0, kWideShort128 = 2000.0, kWideShortParts = 1.05;
 
 // Tile height and K parts.  What a wavefront spends on a K-tile depends on the tile height alone (the weights of its 64
 // columns are dequantised once per K-tile whatever the rows: about 2500 cycles at 256 rows, 1600 at 128, measured
@@ -155,27 +161,27 @@ GemmLaunchShape gemm_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_par
             if (parts != splits) continue;
             const uint32_t all = ((m + bm - 1) / bm) * tiles_n * parts;
             const uint32_t shorts = wide_short_rows(m, bm) ? tiles_n * parts : 0, wgs = all - shorts;
-            // cycles of a workgroup per K-tile, measured under load: 2500 at 256 rows (one workgroup a CU, whole rounds);
-            // 1600 at 128 rows alone on its CU, 2950 for the two that share one (a last round of at most one per CU
-            // runs alone)
+            // cycles of a workgroup per K-tile, measured under load: 2500 at 256 rows (one workgroup a CU, whole rounds; 2050
+            // to 2750 by how many of the CUs are at work); 1600 at 128 rows alone on its CU, 2950 for the two that share one
+            // (a last round of at most one per CU runs alone)
             double cycles;
+            uint32_t rounds, short_rounds = 0;
             if (bm == 256) {
-                cycles = (double)((wgs + cus - 1) / cus) * per * 2500.0;
-                // the short tiles of a cut last row: on the CUs the last round leaves idle, the
-                // others in rounds of their own
-                if (shorts) {
-                    const double each = m % bm <= 64 ? kWideShort64 : kWideShort128;
-                    const uint32_t idle = wgs % cus ? cus - wgs % cus : 0;
-                    const uint32_t beside = idle * (uint32_t)(2500.0 / each);
-                    if (shorts > beside) cycles += (double)((shorts - beside + cus - 1) / cus) * per * each;
-                }
+                rounds = (wgs + cus - 1) / cus;
+                cycles = (double)rounds * per * 2500.0;
+                // the short tiles of a cut last row: on the CUs the last round leaves idle, the others in rounds of their own
+                const uint32_t idle = rounds * cus - wgs;
+                if (shorts > idle) short_rounds = (shorts - idle + cus - 1) / cus;
+                cycles += (double)short_rounds * per * (m % bm <= 64 ? kWideShort64 : kWideShort128);
+                rounds += short_rounds;
             } else {
+                rounds = (wgs + 2 * cus - 1) / (2 * cus);
                 const uint32_t full = wgs / (2 * cus), rest = wgs % (2 * cus);
                 cycles = (double)full * per * 2950.0 + (rest > cus ? per * 2950.0 : rest ? per * 1600.0 : 0.0);
             }
-            const double rounds = bm == 256 ? (double)((wgs + cus - 1) / cus) : (double)((wgs + 2 * cus - 1) / (2 * cus));
             double cost = cycles / 1750.0 + 8.0 * rounds;                       // us at the clock the part holds
             if (parts > 1) cost += 3.0 + (double)(parts + 1) * m * n * 4.0 / 3.5e6;
+            if (parts > 1 && short_rounds) cost *= kWideShortParts;
             if (best == 0 || cost < best) {
                 best = cost;
                 g.bm = bm; g.splits = parts; g.kt_per_split = per;

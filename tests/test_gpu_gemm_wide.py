@@ -254,6 +254,22 @@ def test_short_last_row_tile_of_256_rows_exact(pkg, ctx, m, parts, f16):
     w.destroy()
 
 
+@pytest.mark.parametrize("n,k,x_name,cells", [(16384, 8192, "BF16", [(257, 2), (320, 2)]), (24576, 11008, "BF16", [(384, 1)]),
+                                              (28672, 4096, "F32", [(517, 1), (600, 1), (640, 1)])])
+def test_short_row_tiles_do_not_draw_a_launch_into_more_k_parts(pkg, ctx, n, k, x_name, cells):
+    """The planned shape where a short last row tile takes a round of its own: 256-row tiles in the number of K parts that
+    was measured fastest (four parts at 16384 x 8192 cost 5 to 9 %, at 24576 x 11008 10 %; two parts of gate+up in fp32
+    gain nothing for 119 MB of partial results).  The plan alone: nothing is launched."""
+    fmt = pkg.QuantizationFormatRegistry.format_for_mlx_quantization(4, 64)
+    planes = np.zeros((n, k // 8), np.uint32), np.zeros((n, k // 64), np.uint16), np.zeros((n, k // 64), np.uint16)
+    w = ctx.weight_prepare_mlx(fmt, *planes, pkg.F16, pkg.LAYOUT_PLANES)
+    for m, parts in cells:
+        step = w.plan_prefill_steps(m, x_dtype=getattr(pkg, x_name))[0]
+        tiles = -(-m // 256) * -(-n // 256)
+        assert step.device_kernel.endswith("qgemm_wide_q4_g64") and step.grid[0] == -(-tiles * parts // 8) * 8, (m, step.grid, tiles)
+    w.destroy()
+
+
 def _wrapped(pkg, ctx, group, codes, scales, zeros):
     """Borrowed bf16 planes (mi355q_weight_wrap_planes): the only weights whose scales may be any bf16 number."""
     n, k = codes.shape
