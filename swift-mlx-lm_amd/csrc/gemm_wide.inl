@@ -388,11 +388,15 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
         walk(std::integral_constant<int, TM>{});
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // the lane's number counted again: what the epilogue derives from it is then not shared with the offsets of the loads
-    // above and kept over the K loop, in registers that the 128-row form does not have (it spilled up to two for them)
-    uint32_t all_lanes = ~0u;
-    asm volatile("" : "+s"(all_lanes));
-    const uint32_t lane_e = __builtin_amdgcn_mbcnt_hi(all_lanes, __builtin_amdgcn_mbcnt_lo(all_lanes, 0));
+    // 128 rows: the lane's number counted again.  What the epilogue derives from it is then not shared with the offsets of the
+    // loads above and kept over the K loop, in registers that this form does not have (it spilled up to two for them; a layer
+    // at 128 rows 167.97 -> 167.05 us).  The 256-row form has registers to spare and keeps its numbers.
+    uint32_t lane_e = lane;
+    if constexpr (BM == 128) {
+        uint32_t all_lanes = ~0u;
+        asm volatile("" : "+s"(all_lanes));
+        lane_e = __builtin_amdgcn_mbcnt_hi(all_lanes, __builtin_amdgcn_mbcnt_lo(all_lanes, 0));
+    }
     if (probing) {
         const unsigned long long c1 = __builtin_readcyclecounter(), r1 = __builtin_amdgcn_s_memrealtime();
         if (lane_e == 0) { a.probe[0] = c1 - probe_c0; a.probe[1] = r1 - probe_r0; }
