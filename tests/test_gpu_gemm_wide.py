@@ -15,7 +15,7 @@ import pytest
 
 import kat
 import oracle
-from gpu_util import Case, act_rounded, assert_within_tolerance, seeded_case
+from gpu_util import Case, act_rounded, act_to_device_array, assert_within_tolerance, seeded_case
 from test_gpu_gemm import _tile_edge_sample, bf16_round, run_qgemm
 
 pytestmark = pytest.mark.gpu
@@ -252,6 +252,113 @@ def test_short_last_row_tile_of_256_rows_exact(pkg, ctx, m, parts, f16):
         pkg.Context.probe_wide_shape(0, 0)
     assert np.array_equal(got.astype(np.float64), want)
     w.destroy()
+
+
+def _integers(rng, n, k, group):
+    """A matrix whose every product and sum with small multiples of 1/8 is exact, and the numbers it stands for."""
+    case = Case(4, group, rng.integers(0, 16, (n, k), dtype=np.uint8), rng.choice([0.125, 0.25, 0.5], (n, k // group)),
+                rng.integers(-4, 5, (n, k // group)) * 0.25)
+    return case, case.scales.repeat(group, axis=1) * case.codes + case.zeros.repeat(group, axis=1)
+
+
+def _grid_of_256_row_tiles(m, n, parts):
+    return -(-(-(-m // 256) * -(-n // 256) * parts) // 8) * 8
+
+
+@pytest.mark.parametrize("layout_name,sb_name,group", [("LAYOUT_PLANES", "F16", 64), ("LAYOUT_PLANES", "BF16", 64), ("LAYOUT_PLANES", "F16", 128),
+                                                       ("LAYOUT_PLANES", "BF16", 128), ("LAYOUT_STAF_BLOCKS", "F16", 64),
+                                                       ("LAYOUT_STAF_BLOCKS", "F16", 128)])
+@pytest.mark.parametrize("x_name", ["BF16", "F16", "F32"])
+def test_short_last_row_tile_on_every_layout_group_and_scale_type_exact(pkg, ctx, layout_name, sb_name, group, x_name):
+    """Every 256-row instantiation of the kernel with both short loops (their wait counts depend on the loads of the layout
+    and of the group): edges of the short heights, the shortest K (four K-tiles) and K in two unequal parts, a ragged
+    last column tile.  The planned grid says that 256-row tiles ran."""
+    rng = np.random.default_rng(5000 + group)
+    n, xd = 2 * 256 + 12, getattr(pkg, x_name)
+    for k, parts, rows in ((256, 1, (257, 320, 321, 384)), (64 * 16 * 2 + 256, 2, (257, 384))):
+        case, wq = _integers(rng, n, k, group)
+        w = case.device_weight(ctx, pkg, getattr(pkg, layout_name), getattr(pkg, sb_name))
+        x = rng.integers(-8, 9, (max(rows), k)).astype(np.float32) * 0.125
+        want = x.astype(np.float64) @ wq.T
+        pkg.Context.probe_wide_shape(256, parts)
+        try:
+            for m in rows:
+                say(f"short last tile {layout_name} sb={sb_name} g{group} x={x_name} m={m} k={k} parts={parts}")
+                step = w.plan_prefill_steps(m, x_dtype=xd, flags=wide(pkg))[0]
+                assert step.device_kernel.endswith(f"qgemm_wide_q4_g{group}") and step.grid[0] == _grid_of_256_row_tiles(m, n, parts)
+                got = run_qgemm(ctx, pkg, w, x[:m], pkg.F32, wide(pkg), x_dtype=xd)
+                assert np.array_equal(got.astype(np.float64), want[:m]), (m, k, parts)
+        finally:
+            pkg.Context.probe_wide_shape(0, 0)
+        w.destroy()
+
+
+@pytest.mark.parametrize("layout_name,x_name", [("LAYOUT_PLANES", "BF16"), ("LAYOUT_PLANES", "F32"), ("LAYOUT_STAF_BLOCKS", "F16")])
+def test_short_last_row_tile_of_a_shared_launch_exact(pkg, ctx, layout_name, x_name):
+    """Three matrices of one launch, the last one ragged, K in one part and in two: every short tile belongs to its matrix
+    and its part."""
+    rng = np.random.default_rng(5100)
+    ns, xd = (256, 512, 132), getattr(pkg, x_name)
+    for parts in (1, 2):
+        k = 64 * 16 * parts + 256
+        cases = [_integers(rng, n, k, 64) for n in ns]
+        ws = [c.device_weight(ctx, pkg, getattr(pkg, layout_name), pkg.F16) for c, _ in cases]
+        for m in (257, 321, 517):
+            x = rng.integers(-8, 9, (m, k)).astype(np.float32) * 0.125
+            xdev = ctx.upload(act_to_device_array(x, xd, pkg))
+            outs = [ctx.alloc(m * n * 4) for n in ns]
+            pkg.Context.probe_wide_shape(256, parts)
+            try:
+                say(f"short last tile, shared launch {layout_name} x={x_name} m={m} parts={parts}")
+                plan = pkg.DispatchPlan(ctx)
+                plan.add_batched_linear(ws, xdev, xd, outs, pkg.F32, m, flags=pkg.FLAG_PROBE_WIDE)
+                assert plan.step(0)[0].grid[0] == _grid_of_256_row_tiles(m, 4 * 256, parts)
+                plan.destroy()
+                ctx.batched_qgemm(ws, xdev, xd, outs, pkg.F32, m, flags=pkg.FLAG_PROBE_WIDE)
+                ctx.synchronize()
+            finally:
+                pkg.Context.probe_wide_shape(0, 0)
+            for o, n, (_, wq) in zip(outs, ns, cases):
+                assert np.array_equal(o.download(np.float32, (m, n)).astype(np.float64), x.astype(np.float64) @ wq.T), (m, n, parts)
+                o.free()
+            xdev.free()
+        for w in ws:
+            w.destroy()
+
+
+@pytest.mark.parametrize("layout_name,x_name,group", [("LAYOUT_PLANES", "BF16", 64), ("LAYOUT_PLANES", "F16", 128), ("LAYOUT_STAF_BLOCKS", "BF16", 64)])
+def test_short_last_row_tile_of_a_gated_launch(pkg, ctx, layout_name, x_name, group):
+    """Gate and up as the two fragments of a wavefront: the sums are exact, so the one launch on 256-row tiles equals, bit
+    for bit, the projections on 128-row tiles (which are never short) and the elementwise kernel behind them; a whole and
+    a ragged column tile, 16-bit and fp32 results."""
+    rng = np.random.default_rng(5200 + group)
+    n, k, xd = 128 + 37, 3 * 256, getattr(pkg, x_name)
+    gate, up = (_integers(rng, n, k, group)[0].device_weight(ctx, pkg, getattr(pkg, layout_name), pkg.F16) for _ in range(2))
+    for m in (257, 320, 321, 384):
+        x = rng.integers(-8, 9, (m, k)).astype(np.float32) * 0.125
+        xdev = ctx.upload(act_to_device_array(x, xd, pkg))
+        for yd, dt in ((pkg.F32, np.float32), (xd, np.uint16)):
+            fused, a, b, two = (ctx.alloc(m * n * 4) for _ in range(4))
+            say(f"short last tile, gated launch {layout_name} x={x_name} g{group} m={m} y={yd}")
+            try:
+                pkg.Context.probe_wide_shape(256, 1)
+                plan = pkg.DispatchPlan(ctx)
+                plan.add_gated_mlp(gate, up, xdev, xd, fused, yd, m, flags=pkg.FLAG_PROBE_WIDE)
+                assert plan.step(0)[0].grid[0] == _grid_of_256_row_tiles(m, 2 * n, 1)
+                plan.destroy()
+                ctx.gated_qgemm(gate, up, xdev, xd, fused, yd, m, flags=pkg.FLAG_PROBE_WIDE)
+                pkg.Context.probe_wide_shape(128, 1)
+                for w, y in ((gate, a), (up, b)):
+                    ctx.qgemm(w, xdev, xd, y, yd, m, flags=wide(pkg))
+            finally:
+                pkg.Context.probe_wide_shape(0, 0)
+            ctx.gated_activation(a, b, two, yd, n, m)
+            ctx.synchronize()
+            assert np.array_equal(fused.download(dt)[:m * n], two.download(dt)[:m * n]), (m, yd)
+            for t in (fused, a, b, two):
+                t.free()
+        xdev.free()
+    gate.destroy(); up.destroy()
 
 
 @pytest.mark.parametrize("n,k,x_name,cells", [(16384, 8192, "BF16", [(257, 2), (320, 2)]), (24576, 11008, "BF16", [(384, 1)]),
