@@ -133,16 +133,16 @@ void gemm_wide_force_shape(uint32_t bm, uint32_t splits) {
 // clock than the 2500 cycles below assume (8192 -> 28672 at 270 rows in one part 171 us, charged 191), so splitting K looks
 // better than it is.  Against 186 problems measured at every tile height and number of parts (4096 to 65536 columns, K walks
 // of 4096 to 28672, 128 to 2432 rows) the choice is nowhere more than 1.5 % slower than it was without short tiles, and
-// within 4 % of the fastest shape in all but nine (worst 10 %).  With 1800 / 1900 cycles alone, neither the round's 8 us nor
-// the share, 22 of them went into K parts that were slower than before (8192 -> 16384 at 320 rows 116 us in four parts
-// against 107 in two; 11008 -> 24576 at 384 rows 235 in four against 213 in one).
-constexpr double kWideShort64 = 1800.0, kWideShort128 = 2000.0, kWideShortParts = 1.05;
+// within 4 % of the fastest shape in all but nine (worst 10 %).  With 1800 / 1900 cycles and nothing else, 22 of them went
+// into K parts that were slower than before (8192 -> 16384 at 320 rows 116 us in four parts against 107 in two; 11008 ->
+// 24576 at 384 rows 235 in four against 213 in one).
+constexpr double kWideShort64 = 1400.0, kWideShort128 = 1900.0, kWideShortParts = 1.03;
 
 // Tile height and K parts.  What a wavefront spends on a K-tile depends on the tile height alone (the weights of its 64
 // columns are dequantised once per K-tile whatever the rows: about 2500 cycles at 256 rows, 1600 at 128, measured
 // under load), so 256-row tiles are the efficient ones and K is split into parts where they leave CUs idle: each part
 // writes fp32, a second launch adds the parts (about 3 us and the traffic of splits + 1 result matrices).
-GemmLaunchShape gemm_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_part) {
+static GemmLaunchShape choose_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_part, bool count_short, uint32_t most_parts) {
     const uint32_t cus = chip_cus();
     const uint32_t tiles_n = (n + kWideBN - 1) / kWideBN;
     const uint32_t kt = k / 64;
@@ -155,12 +155,12 @@ GemmLaunchShape gemm_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_par
         if (bm == 256 && m <= 128 && !forced_bm) continue;
         for (uint32_t splits : {1u, 2u, 3u, 4u}) {
             if (one_part ? splits != 1 : forced_splits && splits != forced_splits) continue;
-            if (splits > 1 && (n % 4 || kt / splits < 16)) continue;
+            if (splits > 1 && (n % 4 || kt / splits < 16 || splits > most_parts)) continue;
             const uint32_t per = (kt / 4 + splits - 1) / splits * 4;          // K-tiles a part, a multiple of four
             const uint32_t parts = (kt + per - 1) / per;
             if (parts != splits) continue;
             const uint32_t all = ((m + bm - 1) / bm) * tiles_n * parts;
-            const uint32_t shorts = wide_short_rows(m, bm) ? tiles_n * parts : 0, wgs = all - shorts;
+            const uint32_t shorts = count_short && wide_short_rows(m, bm) ? tiles_n * parts : 0, wgs = all - shorts;
             // cycles of a workgroup per K-tile, measured under load: 2500 at 256 rows (one workgroup a CU, whole rounds; 2050
             // to 2750 by how many of the CUs are at work); 1600 at 128 rows alone on its CU, 2950 for the two that share one
             // (a last round of at most one per CU runs alone)
@@ -195,6 +195,13 @@ GemmLaunchShape gemm_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_par
     g.grid = (((m + g.bm - 1) / g.bm) * tiles_n * g.splits + 7) / 8 * 8;
     g.lds_bytes = kWideStages * g.bm * 128;
     return g;
+}
+
+// With a short last row tile: chosen among the numbers of K parts up to the one that whole tiles would take, so that no
+// launch needs partial results, or more of them, because of the short form.
+GemmLaunchShape gemm_wide_shape(uint32_t m, uint32_t n, uint32_t k, bool one_part) {
+    const GemmLaunchShape whole = choose_wide_shape(m, n, k, one_part, false, 4);
+    return wide_short_rows(m, 256) ? choose_wide_shape(m, n, k, one_part, true, whole.splits) : whole;
 }
 
 // Rows from which this kernel is taken instead of the tiled one (which splits K over workgroups for short M) and of

@@ -361,12 +361,13 @@ def test_short_last_row_tile_of_a_gated_launch(pkg, ctx, layout_name, x_name, gr
     gate.destroy(); up.destroy()
 
 
-@pytest.mark.parametrize("n,k,x_name,cells", [(16384, 8192, "BF16", [(257, 2), (320, 2)]), (24576, 11008, "BF16", [(384, 1)]),
+@pytest.mark.parametrize("n,k,x_name,cells", [(16384, 8192, "BF16", [(257, 2), (320, 2)]), (24576, 11008, "BF16", [(300, 1), (384, 1)]),
                                               (28672, 4096, "F32", [(517, 1), (600, 1), (640, 1)])])
 def test_short_row_tiles_do_not_draw_a_launch_into_more_k_parts(pkg, ctx, n, k, x_name, cells):
     """The planned shape where a short last row tile takes a round of its own: 256-row tiles in the number of K parts that
     was measured fastest (four parts at 16384 x 8192 cost 5 to 9 %, at 24576 x 11008 10 %; two parts of gate+up in fp32
-    gain nothing for 119 MB of partial results).  The plan alone: nothing is launched."""
+    gain nothing for 119 MB of partial results), never more of them than whole tiles would take (one at 24576 x 11008 from
+    289 rows).  The plan alone: nothing is launched."""
     fmt = pkg.QuantizationFormatRegistry.format_for_mlx_quantization(4, 64)
     planes = np.zeros((n, k // 8), np.uint32), np.zeros((n, k // 64), np.uint16), np.zeros((n, k // 64), np.uint16)
     w = ctx.weight_prepare_mlx(fmt, *planes, pkg.F16, pkg.LAYOUT_PLANES)
