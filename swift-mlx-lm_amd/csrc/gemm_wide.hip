@@ -28,7 +28,7 @@
 //   * one barrier per K-tile, in the middle of it: K-tile kt + 1 has landed for everyone, and the stage of K-tile
 //     kt - 1 is free for kt + 3;
 //   * a last 256-row tile of at most 64 or 128 rows copies and multiplies those fragments only, and its workgroups come last,
-//     on the CUs the last round of whole tiles leaves idle (gate+up 2 x 14336 at 517 fp32 rows 322 -> 297 us);
+//     on the CUs the last round of whole tiles leaves idle (gate+up 2 x 14336 at 517 fp32 rows 318-324 -> 294-299 us);
 //   * BM = 256 where that fills the chip (one workgroup per CU, 256 accumulator registers per lane), BM = 128 elsewhere
 //     (two workgroups per CU); where 256-row tiles would leave CUs idle, K goes over workgroups in parts.
 // The kernel text is gemm_wide.inl; this file chooses the shape, launches, and adds the parts of K.

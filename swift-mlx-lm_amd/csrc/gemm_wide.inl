@@ -94,8 +94,8 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
 
     // ---- activations: global -> LDS ---------------------------------------------------------------
     // copy q of wavefront w covers tile rows 8 (4 q + w) .. + 7 of 256 (so that the first copies of all wavefronts are the
-    // rows a short tile needs), 8 (4 w + q) .. of 128 (the registers of that form are full: it spills the other way); lane L lands at row L / 8, position L % 8, and
-    // fetches the chunk that belongs there after the rotation.  Rows past M re-read the last one.
+    // rows a short tile needs), 8 (4 w + q) .. of 128 (whose tiles are never short); lane L lands at row L / 8, position
+    // L % 8, and fetches the chunk that belongs there after the rotation.  Rows past M re-read the last one.
     const uint32_t m_last = a.m - 1 - m0;           // last valid row of the tile
     uint32_t x_off[AQ];
 #pragma unroll
@@ -248,13 +248,14 @@ __global__ __launch_bounds__(256, (BM == 128 ? 2 : 1)) void qgemm_wide_kernel(Wi
         }
     };
     // a quarter of the dequantisation of word w of fragment f: codes 2 p and 2 p + 1 as one packed pair of the
-    // activations' type.  The pieces come in the order p = 0, 2, 1, 3.  A nibble alone in the low seven bits' reach of a
-    // half-word is, read as f16, the (subnormal) number q * 2^-24, or q * 2^-20 a nibble further up, and the mixed-type
-    // fma takes either half of a register as such a number: fma(scale * 2^24, q * 2^-24, bias) is fma(scale, q, bias) bit
-    // for bit (powers of two), with no conversion, where byte extraction plus convert took 22 instructions for eight codes
-    // and this takes 17 (a Llama-3-8B layer's projections at 128 / 2048 bf16 rows 168.5 -> 165.3 / 813 -> 800 us, at 517
-    // fp32 rows 659 -> 643; same bits).  A bf16 scale of 2^104 or more would leave the fp32 range times 2^24 (and give
-    // infinity times code 0): weights that hold one (kWideScalesBf16Any; only borrowed planes can) have their bytes converted.
+    // activations' type.  The pieces come in the order p = 0, 2, 1, 3.  A nibble alone in the low byte of a half-word is,
+    // read as f16, the number q * 2^-24, or q * 2^-20 in the upper half of that byte (subnormal either way: their field has
+    // ten bits), and the mixed-type fma takes either half of a register as such a number: fma(scale * 2^24, q * 2^-24, bias)
+    // is fma(scale, q, bias) bit for bit (powers of two), with no conversion, where byte extraction plus convert took 22
+    // instructions for eight codes and this takes 17 (4096 -> 14336 at 2048 bf16 rows 31.41 M -> 26.99 M vector instructions,
+    // 12.60 M -> 12.19 M busy cycles, 198 -> 194 us; a Llama-3-8B layer's projections at 128 / 2048 rows 174.2 -> 170.8 /
+    // 867.6 -> 854.3; same bits).  A bf16 scale of 2^104 or more would leave the fp32 range times 2^24 (and give infinity
+    // times code 0): weights that hold one (kWideScalesBf16Any; only borrowed planes can) have their bytes converted.
     // piece b of a word is the pair of codes (c0,c1) (c4,c5) (c2,c3) (c6,c7): its place among the operand's four registers
     auto dq_place = [](int b) constexpr { return ((b & 1) << 1) | (b >> 1); };
     uint32_t dq_t[2], dq_u[2];
